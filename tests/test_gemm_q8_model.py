@@ -77,13 +77,15 @@ def act_layout(q, d, qt):
     return y
 
 
-def buf_load(mem, base, nbytes, off, size):
-    """raw buffer load: dwords past the resource read 0; the others stay in mem"""
+def buf_load(mem, base, nbytes, voff, soff, size):
+    """raw buffer load: dwords whose vector offset is past the resource read 0, the others must
+    lie in mem. The scalar offset moves the address and is no part of the check."""
     out = np.zeros(size, np.uint8)
-    n = max(0, min(size, (nbytes - off) & ~3))
+    n = max(0, min(size, (nbytes - voff) & ~3))
     if n:
-        assert 0 <= base + off and base + off + n <= mem.size
-        out[:n] = mem[base + off:base + off + n]
+        at = base + voff + soff
+        assert 0 <= at and at + n <= mem.size
+        out[:n] = mem[at:at + n]
     return out
 
 
@@ -119,7 +121,7 @@ def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0):
     pitch = sd + 1
     rows, toks = min(N - n0, BN), min(M - m0, 32 * mt)
     acc = np.zeros((BN, 32 * mt), np.float32)
-    for s in range(s0, s1):
+    for s in range(s0, s1 + 2):  # the pipeline requests two stages past its last: nothing is read
         lw = np.zeros(BN * pitch, np.uint32)
         la = np.zeros(32 * mt * ROW, np.uint8)
         ld = np.zeros(256 * 8, np.uint8)
@@ -130,17 +132,21 @@ def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0):
                 r, w = divmod(tid + 256 * u, npc)
                 if r >= BN:
                     continue  # writes behind the rows
-                off = r * rb + 8 * w + s * sd * 4 if r < rows else 0x80000000
+                off = r * rb + 8 * w if r < rows else 0x80000000
                 wpos = pitch * r + 2 * w
                 assert not wrote[wpos:wpos + 2].any()  # no dword has two writers
                 wrote[wpos:wpos + 2] = True
-                lw[wpos:wpos + 2] = buf_load(W, n0 * rb, rows * rb, off, 8).view(np.uint32)
+                lw[wpos:wpos + 2] = buf_load(W, n0 * rb + s * sd * 4, rows * rb - s * sd * 4 if s < s1 else 0, off,
+                                             0, 8).view(np.uint32)
             apos = (tid >> 3) * ROW + (((tid & 7) ^ ((tid >> 3) & 7)) << 4)
             for i in range(mt):
-                la[apos + 4096 * i:apos + 4096 * i + 16] = buf_load(A, (s * M + m0) * ROW, toks * ROW,
-                                                                    16 * tid + 4096 * i, 16)
-            v = buf_load(A, ns * M * ROW + (s * M + m0) * 8, toks * 8, 8 * tid, 8)
+                la[apos + 4096 * i:apos + 4096 * i + 16] = buf_load(A, (s * M + m0) * ROW, toks * ROW * (s < s1),
+                                                                    16 * tid + 4096 * i, 0, 16)
+            v = buf_load(A, ns * M * ROW + (s * M + m0) * 8, toks * 8 * (s < s1), 8 * tid, 0, 8)
             ld[8 * tid:8 * tid + 8] = v
+        if s >= s1:
+            assert not lw.any() and not la.any() and not ld.any()
+            continue
         for wave in range(4):
             q, d = {}, {}
             for lane in range(64):
