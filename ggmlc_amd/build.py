@@ -2,7 +2,7 @@
 
 Every .hip file under csrc/ is compiled by hipcc to an object in
 ggmlc_amd/_build/ (parallel), then linked into ggmlc_amd/libgq.so. The benchmark's
-measurement aids under bench_csrc/ (the streaming-read probe) are linked into their
+measurement aids under bench_csrc/ (the streaming-read probe; the launch plans) are linked into their
 own ggmlc_amd/libgqbench.so, outside libgq's ABI.
 """
 

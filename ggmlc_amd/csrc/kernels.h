@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.h"
+#include "plans.h"
 
 namespace gq {
 
@@ -118,13 +119,9 @@ int gemm(int type, const uint8_t* W, int64_t N, int64_t K, const uint16_t* A, in
 // gemm_q8.hip — dst[m * ldd + n] (+ bias[n]) for more than GEMM_I8_MAX_M rows on int8 MFMA,
 // from act_prep_q8's layout, for weights whose rows are 4-byte aligned (gemm_q8_ok: K % 64
 // == 0; odd block counts leave rows only 2-byte aligned and take gemm)
-struct GemmQ8Plan {
-    int mt;       // 32-token tiles per workgroup
-    int ks, sps;  // K splits and stages per split
-};
 bool gemm_q8_ok(int64_t K);
 size_t gemm_q8_act_bytes(int64_t K, int64_t M);
-GemmQ8Plan gemm_q8_plan(int64_t N, int64_t K, int64_t M, size_t part_bytes);  // partials within part_bytes
+GemmQ8Plan gemm_q8_plan(int type, int64_t N, int64_t K, int64_t M, size_t part_bytes);  // partials within part_bytes
 int gemm_q8(int type, const uint8_t* W, int64_t N, int64_t K, const uint8_t* A, int64_t M, float* dst, int64_t ldd,
             float* part, size_t part_bytes, hipStream_t s, const float* bias = nullptr);
 

@@ -5,8 +5,12 @@ block formula."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
+
+from test_gemm_addressing import launches
 
 QK, BN, SBLK, ROW = 32, 128, 4, 128
 Q8, Q4 = 8, 2
@@ -26,38 +30,26 @@ def part_room(N, K, M):
     return _lib.load().gq_mul_mat_workspace_size(w, x) - cdiv(cdiv(K, ROW) * M * (ROW + 8), 256) * 256
 
 
-def fp16_chain(N, K, M, ncu=256):
-    """blocks per split plus splits of gemm.hip's gemm_plan, whose K steps are 2 blocks"""
-    bm = 128 if (M > 64 and cdiv(N, BN) >= 16) or cdiv(N, BN) * cdiv(M, 128) >= ncu else 64
-    tiles, nk, ks = cdiv(N, BN) * cdiv(M, bm), cdiv(K, 64), 1
-    if tiles < ncu:
-        ks = max(min(cdiv((1 if bm == 128 else 2) * ncu, tiles), nk // 4, 16), 1)
-    spk = cdiv(nk, ks)
-    return 2 * spk + cdiv(nk, spk)
+def bench_lib():
+    """libgqbench.so, which answers the library's own plans without a device"""
+    from ggmlc_amd import build
+
+    lib = ctypes.CDLL(str(build.BENCH_LIB))
+    lib.gqbench_gemm_q8_plan.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [ctypes.c_size_t, ctypes.c_int64,
+                                                                                 ctypes.POINTER(ctypes.c_int)]
+    lib.gqbench_gemm_q8_plan.restype = None
+    lib.gqbench_fp16_pair_chain.argtypes = [ctypes.c_int64] * 4
+    lib.gqbench_fp16_pair_chain.restype = ctypes.c_double
+    return lib
 
 
-def plan(N, K, M, ncu=256):
-    """gemm_q8_plan: (32-token tiles per workgroup, K splits, stages per split)"""
-    ns, slab, room = cdiv(K, ROW), 4 * M * N, part_room(N, K, M)
+def plan(qt, N, K, M, ncu=256):
+    """plan_gemm_q8: (32-token tiles per workgroup, K splits, stages per split, stages per segment)"""
+    room, out = part_room(N, K, M), (ctypes.c_int * 4)()
     assert room >= 0
-    most = min(1 + room // slab, max(1, ns // 3), 16)
-    most = cdiv(ns, cdiv(ns, most))
-    bound = max(20, fp16_chain(N, K, M), min(4 * cdiv(ns, z) + z for z in range(1, most + 1)))
-    best = None
-    for mt in range(min(4, cdiv(M, 32)), 0, -1):
-        one, two = 0.56 + 0.245 * mt, 0.53 + 0.485 * mt
-        for z in range(1, most + 1):
-            sps = cdiv(ns, z)
-            if cdiv(ns, sps) != z or 4 * sps + z > bound:
-                continue
-            load = cdiv(cdiv(N, BN) * cdiv(M, 32 * mt) * z, ncu)
-            us = sps * (0.5 * load if mt == 1 and load > 1 else load // 2 * two + (load & 1) * one)
-            us += (3.0 * ((load - 1) // 2) if mt > 1 else 0.0) + (5.0 + slab * 2 * z / 6e6 if z > 1 else 0.0)
-            if best is None or us < best[0]:
-                best = us, mt, z, sps
-    _, mt, ks, sps = best
-    assert (ks - 1) * slab <= room  # split 0 stands in dst
-    return mt, ks, sps
+    bench_lib().gqbench_gemm_q8_plan(qt, N, K, M, room, ncu, out)
+    assert (out[1] - 1) * 4 * M * N <= room  # split 0 stands in dst
+    return tuple(out)
 
 
 def act_layout(q, d, qt):
@@ -114,13 +106,14 @@ def weight_operand(lds, wr, h, j, qt):
     return np.array(q, np.uint32).view(np.int8), np.array(pr, np.uint32).view(np.float16)
 
 
-def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0):
-    """acc [BN, 32 mt] of one workgroup (before the epilogue's power of two)"""
+def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, seg, n0, m0):
+    """sums [BN, 32 mt] of one workgroup (before the epilogue's power of two): segments of seg
+    stages, each from zero, one after the other"""
     nb, ns = K // QK, cdiv(K, ROW)
     rb, sd = nb * BB[qt], BB[qt]
     pitch = sd + 1
     rows, toks = min(N - n0, BN), min(M - m0, 32 * mt)
-    acc = np.zeros((BN, 32 * mt), np.float32)
+    acc, total = np.zeros((BN, 32 * mt), np.float32), None
     for s in range(s0, s1 + 2):  # the pipeline requests two stages past its last: nothing is read
         lw = np.zeros(BN * pitch, np.uint32)
         la = np.zeros(32 * mt * ROW, np.uint8)
@@ -147,6 +140,8 @@ def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0):
         if s >= s1:
             assert not lw.any() and not la.any() and not ld.any()
             continue
+        if s > s0 and (s - s0) % seg == 0:
+            total, acc = acc if total is None else acc + total, np.zeros_like(acc)
         for wave in range(4):
             q, d = {}, {}
             for lane in range(64):
@@ -170,7 +165,7 @@ def run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0):
                     assert abs(S).max() < 2**24  # exact as fp32
                     sl = (slice(32 * wave, 32 * wave + 32), slice(32 * i, 32 * i + 32))
                     acc[sl] = (S * P + acc[sl]).astype(np.float32)
-    return acc
+    return acc if total is None else acc + total
 
 
 SHAPES = [(130, 64, 17), (100, 192, 33), (129, 960, 70), (33, 576, 100), (256, 128, 130), (5, 1152, 21),
@@ -197,7 +192,7 @@ def test_data_path(qt, N, K, M):
     assert A.size == cdiv(K, ROW) * M * (ROW + 8)  # gemm_q8_act_bytes
     want = np.einsum("nbj,mbj,nb,mb->mn", qw.astype(np.float64), qx.astype(np.float64), dw.astype(np.float64),
                      dx.astype(np.float64))
-    mt, ks, sps = plan(N, K, M)
+    mt, ks, sps, seg = plan(qt, N, K, M)
     ns = cdiv(K, ROW)
     n_tiles, m_tiles = cdiv(N, BN), cdiv(M, 32 * mt)
     out = np.full((ks, M, N), np.nan, np.float32)
@@ -213,7 +208,7 @@ def test_data_path(qt, N, K, M):
         seen.add((z, n0, m0))
         s0, s1 = z * sps, min(ns, z * sps + sps)
         assert s0 < s1
-        acc = run_workgroup(qt, N, K, M, W, A, mt, s0, s1, n0, m0)
+        acc = run_workgroup(qt, N, K, M, W, A, mt, s0, s1, seg, n0, m0)
         for wave in range(4):
             for lane in range(64):
                 c, h = lane & 31, lane >> 5
@@ -236,8 +231,30 @@ def test_data_path(qt, N, K, M):
 @pytest.mark.parametrize("N,K,M", [(4096, 4096, 512), (22016, 4096, 100), (4096, 11008, 17), (49152, 960, 333),
                                    (1536, 8960, 300), (2048, 1536, 40), (151936, 1536, 512), (32, 64, 1000)])
 def test_plan_covers_k_once(N, K, M):
-    mt, ks, sps = plan(N, K, M)
-    ns = cdiv(K, ROW)
-    assert 1 <= mt <= 4 and ks >= 1 and (ks - 1) * sps < ns <= ks * sps
-    for qt in (Q8, Q4):  # two workgroups' double-buffered stages fit a CU's LDS
+    for qt in (Q8, Q4):
+        mt, ks, sps, seg = plan(qt, N, K, M)
+        ns = cdiv(K, ROW)
+        assert 1 <= mt <= 4 and ks >= 1 and (ks - 1) * sps < ns <= ks * sps and 1 <= seg <= sps
+        # two workgroups' double-buffered stages fit a CU's LDS
         assert 2 * 2 * (BN * (BB[qt] + 1) * 4 + 16 + mt * 32 * ROW + 256 * 8) <= 160 * 1024
+
+
+def chain(K, ks, sps, seg):
+    """blocks per fp32 chain + chains a sum goes through, which its squared error grows with"""
+    return min(4 * seg, K // QK) + cdiv(sps, seg) + ks - 1
+
+
+@pytest.mark.parametrize("K", [64, 256, 320, 576, 832, 960, 1536, 2560, 4096, 8960, 11008, 16384])
+def test_plan_rounds_no_more_than_the_fp16_pairs(K):
+    """the sums are no longer than in the order of gemm.hip's plan (a last partial round of tiles
+    counts by its share of the rows); Q8_0, whose block sums are rounded there, 6 blocks more"""
+    lib = bench_lib()
+    for N in (96, 960, 1536, 1600, 2048, 4096, 5120, 12288, 17920, 22016, 32000):
+        for M in (5, 17, 40, 64, 65, 100, 160, 256, 300, 400, 512, 1000):
+            old = 0.0
+            for n, _, ks, spk in launches(N, K, M):
+                old += n / N * (min(2 * spk, K // QK) + ks)
+            assert abs(lib.gqbench_fp16_pair_chain(N, K, M, 256) - old) < 1e-9, (N, M)
+            for qt in (Q8, Q4):
+                _, ks, sps, seg = plan(qt, N, K, M)
+                assert chain(K, ks, sps, seg) <= old + (6 if qt == Q8 else 0), (qt, N, M)
