@@ -104,16 +104,23 @@ class Workspace:
         return self.buf.data_ptr(), self.buf.numel()
 
 
-_default_ws: dict[int, Workspace] = {}
+class _CallScratch:
+    """The scratch of one call without a workspace of its own: from torch's allocator, so
+    calls on different streams (and threads) never share it, and inside a graph capture it
+    belongs to that graph. The caller keeps the object until the call has been launched."""
+
+    def __init__(self):
+        self.buf = None
+
+    def get(self, nbytes: int) -> tuple[int, int]:
+        if nbytes == 0:
+            return 0, 0
+        self.buf = torch.empty(nbytes, dtype=torch.uint8, device=torch.device("cuda", torch.cuda.current_device()))
+        return self.buf.data_ptr(), nbytes
 
 
-def _ws(ws: Workspace | None) -> Workspace:
-    if ws is not None:
-        return ws
-    dev = torch.cuda.current_device()
-    if dev not in _default_ws:
-        _default_ws[dev] = Workspace(torch.device("cuda", dev))
-    return _default_ws[dev]
+def _ws(ws: Workspace | None) -> Workspace | _CallScratch:
+    return ws if ws is not None else _CallScratch()
 
 
 class separate_attn_merge:
@@ -174,7 +181,8 @@ def mul_mat(w: QWeight, x: torch.Tensor, out: torch.Tensor | None = None,
     L = _lib.load()
     a, b, d = w.desc(), _desc(x), _desc(out)
     need = L.gq_mul_mat_workspace_size(a, b)
-    ptr, size = _ws(ws).get(need)
+    ws = _ws(ws)
+    ptr, size = ws.get(need)
     check(L.gq_mul_mat(a, b, d, ptr, size, _stream()))
     return out
 
@@ -268,7 +276,8 @@ def mul_mat_fused(w: QWeight, x: torch.Tensor, out: torch.Tensor | None = None, 
     L, wd, xd = _lib.load(), w.desc(), _desc(x)
     need = L.gq_mul_mat_fused_workspace_size(wd, xd, ctypes.byref(f))
     if need:
-        f.workspace, f.workspace_bytes = _ws(ws).get(need)
+        ws = _ws(ws)
+        f.workspace, f.workspace_bytes = ws.get(need)
     check(L.gq_mul_mat_fused(wd, xd, od, ctypes.byref(f), _stream()))
     del keep
     return out
@@ -298,7 +307,8 @@ def flash_attn_ext(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: torc
     qd, kd, vd, od = _desc(q), _desc(k), _desc(v), _desc(out)
     md = _desc(mask) if mask is not None else None
     need = L.gq_flash_attn_ext_workspace_size(qd, kd)
-    ptr, size = _ws(ws).get(need)
+    ws = _ws(ws)
+    ptr, size = ws.get(need)
     check(L.gq_flash_attn_ext(qd, kd, vd, md, scale, max_bias, logit_softcap, od, ptr, size, _stream()))
     return out
 
@@ -318,7 +328,8 @@ def flash_attn_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
     L = _lib.load()
     qd, kd, vd, od = _desc(q), _desc(k_pool), _desc(v_pool), _desc(out)
     need = L.gq_flash_attn_paged_workspace_size(qd, kd, max_len, page_size)
-    ptr, size = _ws(ws).get(need)
+    ws = _ws(ws)
+    ptr, size = ws.get(need)
     if out_q8 is not None:
         check(L.gq_flash_attn_paged_q8(qd, kd, vd, _desc(page_table), _desc(seq_len), page_size, max_len, scale, od,
                                        out_q8.data_ptr(), ptr, size, _stream()))

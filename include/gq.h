@@ -256,7 +256,9 @@ int gq_set_rows(gq_tensor* a, const gq_tensor* b, const gq_tensor* c, int32_t* n
  * arrival counters that belong to the launch's stream (16 streams per process have
  * their own; launches on further streams merge in a second launch), so calls on
  * different streams may overlap; graphs captured on one stream must not be replayed
- * concurrently. */
+ * concurrently. The workspace holds the splits' partials between the launches of one call:
+ * decode calls and, where their query tiles leave CUs idle, prompt calls write it (head dims
+ * 64 and 128 from n_kv = 1024 on), so calls that may overlap take workspaces of their own. */
 size_t gq_flash_attn_ext_workspace_size(const gq_tensor* q, const gq_tensor* k);
 int gq_flash_attn_ext(const gq_tensor* q, const gq_tensor* k, const gq_tensor* v,
                       const gq_tensor* mask, float scale, float max_bias, float logit_softcap,
@@ -271,7 +273,8 @@ int gq_flash_attn_ext(const gq_tensor* q, const gq_tensor* k, const gq_tensor* v
  * (its address is looked up by gq_init, or by the first call on the device). A
  * shape whose partials need more (gq_flash_attn_ext_workspace_size) returns
  * GQ_ERR_WORKSPACE before anything launches. Calls share the array, so two calls
- * that overlap on one device race: issue them on one stream. */
+ * that overlap on one device race, decode and prompt calls alike: issue them on one
+ * stream. */
 #define GQ_ATTN_SCRATCH_BYTES ((size_t)16 << 20)
 int gq_flash_attn_ext_noalloc(const gq_tensor* q, const gq_tensor* k, const gq_tensor* v,
                               const gq_tensor* mask, float scale, float max_bias, float logit_softcap,

@@ -985,3 +985,34 @@ def test_flash_attn_decode_on_two_streams(Hq, Hkv, D, pos, ctx):
     for i in range(2):
         for o in outs[i]:
             assert torch.equal(o, alone[i]), i
+
+
+@pytest.mark.parametrize("call", ["prompt", "decode", "product"])
+def test_calls_without_a_workspace_on_two_streams(call):
+    """Calls that name no workspace, issued on two streams at once: a prompt whose keys are split
+    over workgroups, a decode with split keys and a product with K splits each write partials, and
+    every output has the bits of the same call run alone."""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(5)
+    rn = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    runs = []
+    for _ in range(2):
+        if call == "product":
+            w, x = ops.quantize_weights(rn(4096, 4096) * 0.02, O.Q8_0), rn(100, 4096)
+            runs.append(lambda w=w, x=x: ops.mul_mat(w, x))
+        else:
+            S, n = (128, 3072) if call == "prompt" else (1, 4096)
+            q, k, v = rn(12, S, 128), rn(2, n, 128).to(torch.float16), rn(2, n, 128).to(torch.float16)
+            runs.append(lambda q=q, k=k, v=v: ops.flash_attn_ext(q, k, v, None, 0.1))
+    alone = [r() for r in runs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = [[], []]
+    for _ in range(24):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(runs[i]())
+    torch.cuda.synchronize()
+    for i in range(2):
+        for o in outs[i]:
+            assert torch.equal(o, alone[i]), i
