@@ -560,7 +560,8 @@ __device__ __forceinline__ float merge_splits_ag(const float* base, int64_t stri
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-// Prefill attention on the matrix cores (v_mfma_f32_16x16x32_f16), no ALiBi / softcap.
+// Prefill attention on the matrix cores (v_mfma_f32_16x16x32_f16), no ALiBi / softcap, for the
+// masks that k_attn_pre does not read (pre_ok: not 8-byte aligned, n_kv % 4 != 0, 2 GiB and more).
 // A workgroup owns 16 WQ query vectors of one kv head (WQ waves x 16), walks the KV range
 // in blocks of 64 keys staged in LDS (K as [key][dim], V transposed to [dim][key]),
 // and keeps an online softmax per query in registers:
@@ -662,38 +663,20 @@ __global__ __launch_bounds__(64 * WQ) void k_attn_mma(AttnArgs a, int G, int NQ,
     };
 
     const int nblk = (int)((a.n_kv + BKV - 1) / BKV);
-    // Mask values of this lane's keys (16 t + 4 g + r) of a block: one 8-byte raw buffer
-    // load per t, issued with the block's K/V prefetch (rows past S and missing masks
-    // read 0 without a fetch; keys past n_kv and lanes without a query become -inf when
-    // unpacked). With n_kv % 4 == 0 every 4-key group of a row lies inside the row;
-    // other shapes, and row strides that are not a multiple of 8 bytes, take 2-byte loads.
-    const bool m8 = a.mask && a.mnb1 % 8 == 0 && a.n_kv % 4 == 0 && (reinterpret_cast<uintptr_t>(a.mask) & 7) == 0;
-    const __amdgpu_buffer_rsrc_t mrs = [&] {
-        const uint64_t base = reinterpret_cast<uint64_t>(a.mask);
-        const int64_t bytes = m8 ? a.S * a.mnb1 : 0;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
-        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
-        const uint32_t n = (uint32_t)(bytes > 0x7fffffff ? 0x7fffffff : bytes);
-        return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0,
-                                                 (int)__builtin_amdgcn_readfirstlane(n), 0x00020000);
-    }();
-    const uint8_t* mrow = a.mask && qok ? reinterpret_cast<const uint8_t*>(a.mask) + qi * a.mnb1 : nullptr;
+    // Mask values of this lane's keys (16 t + 4 g + r) of a block, fetched with the block's K/V:
+    // 2-byte loads, which any alignment and size of the mask takes (keys past n_kv and lanes
+    // without a query become -inf when unpacked)
+    const uint16_t* mrow = qok ? reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(a.mask) + qi * a.mnb1)
+                               : nullptr;
     auto load_mask = [&](int64_t c0, uint32_t (&mw)[4][2]) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int64_t key = c0 + 16 * t + 4 * g;
-            if (m8) {
-                const uint32_t off = qok && key < a.n_kv ? (uint32_t)(qi * a.mnb1 + key * 2) : 0x80000000u;
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(mrs, (int)off, 0, 0);
-                mw[t][0] = v[0];
-                mw[t][1] = v[1];
-            } else {
-                uint16_t h[4];
+            uint16_t h[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) h[r] = mrow && key + r < a.n_kv ? reinterpret_cast<const uint16_t*>(mrow)[key + r] : 0;
-                mw[t][0] = h[0] | ((uint32_t)h[1] << 16);
-                mw[t][1] = h[2] | ((uint32_t)h[3] << 16);
-            }
+            for (int r = 0; r < 4; ++r) h[r] = mrow && key + r < a.n_kv ? mrow[key + r] : 0;
+            mw[t][0] = h[0] | ((uint32_t)h[1] << 16);
+            mw[t][1] = h[2] | ((uint32_t)h[3] << 16);
         }
     };
     auto mask_val = [&](const uint32_t (&mw)[4][2], int64_t c0, int t, int r) -> float {

@@ -89,3 +89,54 @@ def test_masks(Hq, Hkv, S, n_kv):
     run(Hq, Hkv, 128, S, n_kv, m)
     m[S // 2] = float("-inf")  # and one with nothing at all: zeros
     run(Hq, Hkv, 128, S, n_kv, m)
+
+
+def masks(S, n_kv):
+    """causal, banded, -inf holes, finite biases, one key no wave's first lane sees, a row without an
+    unmasked key, one without any"""
+    i, j = torch.arange(S, device=DEV)[:, None], torch.arange(n_kv, device=DEV)[None]
+    yield causal(S, n_kv, n_kv - S)
+    yield torch.where((j - i).abs() < 20, 0.0, -32768.0).to(torch.float16)
+    yield torch.where((i * 7 + j * 13) % 5 == 0, 0.0, float("-inf")).to(torch.float16)
+    yield (-0.01 * (i - j).abs()).to(torch.float16)
+    m = causal(S, n_kv, 3)
+    m[S // 2 + 1, n_kv - 2] = 0.0
+    yield m
+    m = causal(S, n_kv, 5)
+    m[S // 3] = -32768.0
+    m[S // 2] = float("-inf")
+    yield m
+
+
+def shifted(m):
+    """the mask at an address that is not 8-byte aligned"""
+    b = torch.empty(m.numel() + 1, dtype=m.dtype, device=DEV)[1:].view(m.shape)
+    return b.copy_(m)
+
+
+def odd_rows(m):
+    """the mask's rows an odd number of values apart"""
+    return torch.empty((m.shape[0], m.shape[1] + 1 + m.shape[1] % 2), dtype=m.dtype, device=DEV)[:, :-1][
+        :, :m.shape[1]].copy_(m)
+
+
+def past_2gib(m):
+    """the mask's rows spread over more than 2 GiB"""
+    step = 3 * 2**29 // m.shape[0] // 8 * 8  # values from row to row: a third of the rows behind 2 GiB
+    b = torch.empty(step * (m.shape[0] - 1) + m.shape[1], dtype=m.dtype, device=DEV)
+    assert 2 * (b.numel() - m.shape[1]) > 2**31 + 2**29
+    return b.as_strided(m.shape, (step, 1)).copy_(m)
+
+
+# tiles of 32 and of 64 query vectors
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv,S,n_kv", [(4, 2, 70, 300), (32, 32, 300, 304)])
+def test_masks_the_split_kernel_does_not_read(Hq, Hkv, S, n_kv, D):
+    """k_attn_mma: masks not 8-byte aligned, n_kv % 4 != 0, 2 GiB and more"""
+    for m in masks(S, n_kv):
+        run(Hq, Hkv, D, S, n_kv, shifted(m))
+        run(Hq, Hkv, D, S, n_kv, odd_rows(m))
+    for n in (n_kv + 1, n_kv + 3):
+        for m in masks(S, n):
+            run(Hq, Hkv, D, S, n, m)
+    run(Hq, Hkv, D, S, n_kv, past_2gib(causal(S, n_kv, n_kv - S)))
