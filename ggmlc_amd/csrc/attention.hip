@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void k_attn_dec(AttnArgs a, int G, int nq, int
     const int64_t r0 = r_begin + wave * RPI + grp;
     auto rsrc = [&](const void* p, int64_t nb2, int64_t nb1) {
         const uint64_t base = reinterpret_cast<uint64_t>(p) + (uint64_t)(hk * nb2);
-        const int64_t bytes = a.n_kv * nb1;
+        const int64_t bytes = (a.n_kv - 1) * nb1 + D * 2;  // (rows may overlap: any nb1)
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
         const uint32_t n = (uint32_t)(bytes > 0x7fffffff ? 0x7fffffff : bytes);
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(64 * WQ) void k_attn_mma(AttnArgs a, int G, int NQ,
     // K/V rows of this kv head as raw buffers over [0, n_kv): rows past n_kv read 0
     auto rsrc = [&](const void* p, int64_t nb2, int64_t nb1) {
         const uint64_t base = reinterpret_cast<uint64_t>(p) + (uint64_t)(hk * nb2);
-        const int64_t bytes = a.n_kv * nb1;
+        const int64_t bytes = (a.n_kv - 1) * nb1 + D * 2;  // (rows may overlap: any nb1)
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
         const uint32_t n = (uint32_t)(bytes > 0x7fffffff ? 0x7fffffff : bytes);
@@ -876,11 +876,11 @@ __global__ __launch_bounds__(512, 1) void k_attn_pre(AttnArgs a, int G, int NQ, 
         return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0,
                                                  (int)__builtin_amdgcn_readfirstlane(n), 0x00020000);
     };
-    // K/V rows of this kv head over [0, n_kv), mask rows over [0, S): past them loads read 0
-    // without a fetch
-    const __amdgpu_buffer_rsrc_t krs = rsrc(a.k, hk * a.knb2, a.n_kv * a.knb1);
-    const __amdgpu_buffer_rsrc_t vrs = rsrc(a.v, hk * a.vnb2, a.n_kv * a.vnb1);
-    const __amdgpu_buffer_rsrc_t mrs = rsrc(a.mask, 0, a.mask ? a.S * a.mnb1 : 0);
+    // K/V rows of this kv head over [0, n_kv), mask rows over [0, S), to the end of the last row
+    // (rows may overlap: a mask row of stride 0 serves every query): past it loads read 0 without a fetch
+    const __amdgpu_buffer_rsrc_t krs = rsrc(a.k, hk * a.knb2, (a.n_kv - 1) * a.knb1 + D * 2);
+    const __amdgpu_buffer_rsrc_t vrs = rsrc(a.v, hk * a.vnb2, (a.n_kv - 1) * a.vnb1 + D * 2);
+    const __amdgpu_buffer_rsrc_t mrs = rsrc(a.mask, 0, a.mask ? (a.S - 1) * a.mnb1 + a.n_kv * 2 : 0);
     const int nblk = (int)((a.n_kv + 31) / 32);
     const int n_kv = (int)a.n_kv;
 
@@ -1284,7 +1284,7 @@ __global__ __launch_bounds__(256) void k_attn_dec_mma(AttnArgs a, int G, int n_s
 
     auto rsrc = [&](const void* p, int64_t nb2, int64_t nb1) {
         const uint64_t base = reinterpret_cast<uint64_t>(p) + (uint64_t)(hk * nb2);
-        const int64_t bytes = a.n_kv * nb1;
+        const int64_t bytes = (a.n_kv - 1) * nb1 + D * 2;  // (rows may overlap: any nb1)
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
         const uint32_t n = (uint32_t)(bytes > 0x7fffffff ? 0x7fffffff : bytes);
@@ -1492,7 +1492,7 @@ bool pre_ok(const AttnArgs& a) {
     if (!mma_ok(a)) return false;
     if (!a.mask) return true;
     return a.mnb1 % 8 == 0 && a.n_kv % 4 == 0 && (reinterpret_cast<uintptr_t>(a.mask) & 7) == 0 &&
-           a.S * a.mnb1 < 0x7fff0000LL;
+           (a.S - 1) * a.mnb1 + a.n_kv * 2 < 0x7fff0000LL;
 }
 
 // Key splits of k_attn_pre over workgroups (one workgroup fills a CU): as many as fill the CUs

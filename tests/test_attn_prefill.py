@@ -140,3 +140,12 @@ def test_masks_the_split_kernel_does_not_read(Hq, Hkv, S, n_kv, D):
         for m in masks(S, n):
             run(Hq, Hkv, D, S, n, m)
     run(Hq, Hkv, D, S, n_kv, past_2gib(causal(S, n_kv, n_kv - S)))
+
+
+@pytest.mark.parametrize("Hq,Hkv,S,n_kv", [(4, 2, 70, 300), (32, 32, 300, 304), (12, 2, 70, 2048)])
+def test_mask_rows_that_overlap(Hq, Hkv, S, n_kv):
+    """one mask row for every query, and rows that start one 8-byte step after another"""
+    j = torch.arange(n_kv, device=DEV)
+    run(Hq, Hkv, 128, S, n_kv, torch.where(j % 3 == 1, 0.0, -32768.0).to(torch.float16)[None].expand(S, n_kv))
+    b = torch.where(torch.arange(n_kv + 4 * S, device=DEV) % 7 < 3, 0.0, -32768.0).to(torch.float16)
+    run(Hq, Hkv, 128, S, n_kv, b.as_strided((S, n_kv), (4, 1)))
