@@ -84,6 +84,8 @@ def test_masks(Hq, Hkv, S, n_kv):
     late = torch.where((j > n_kv - 40) & (j <= n_kv - 40 + i), 0.0, -32768.0)  # row 0 sees nothing,
     late[0, n_kv - 1] = 0.0  # the others one split's keys only
     run(Hq, Hkv, 128, S, n_kv, late.to(torch.float16))
+    one = torch.where((j - 37 * i) % n_kv == 0, 0.0, -32768.0)  # one key per row, all over the blocks
+    run(Hq, Hkv, 128, S, n_kv, one.to(torch.float16))
     m = causal(S, n_kv, 5)
     m[S // 3] = -32768.0  # one row without an unmasked key: uniform weights plus the scores
     run(Hq, Hkv, 128, S, n_kv, m)
