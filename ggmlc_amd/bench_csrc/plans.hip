@@ -12,3 +12,9 @@ extern "C" void gqbench_gemm_q8_plan(int type, int64_t N, int64_t K, int64_t M, 
 extern "C" double gqbench_fp16_pair_chain(int64_t N, int64_t K, int64_t M, int64_t ncu) {
     return gq::fp16_pair_chain(N, K, M, ncu);
 }
+
+// out: 32-query sub-tiles per workgroup, key splits over workgroups
+extern "C" void gqbench_attn_pre_plan(int64_t NQ, int64_t Hkv, int64_t n_kv, int64_t most, int* out) {
+    const gq::AttnPrePlan p = gq::plan_attn_pre(NQ, Hkv, n_kv, most);
+    out[0] = p.nqw, out[1] = p.ks;
+}

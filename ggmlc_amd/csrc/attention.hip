@@ -1526,17 +1526,8 @@ bool pre_ok(const AttnArgs& a) {
            (a.S - 1) * a.mnb1 + a.n_kv * 2 < 0x7fff0000LL;
 }
 
-// Key splits of k_attn_pre over workgroups (one workgroup fills a CU): as many as fill the CUs
-// where each wave would otherwise walk 4 blocks of 32 keys or more, and keeps 2; at most
-// `most`, the splits the caller's workspace holds. The merge is a launch of its own (~4 us).
-int pre_splits(int64_t wgs, int64_t nblk, int nkw, int64_t most) {
-    const int64_t per_wave = nblk / nkw;
-    if (per_wave < 4) return 1;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({256 / wgs, per_wave / 2, most, 8}));
-}
-
 template <int D, int NQW>
-int launch_pre(const AttnArgs& a, int G, int NQ, int q_f16, int q_al, float* part, int64_t most, hipStream_t s) {
+int launch_pre(const AttnArgs& a, int G, int NQ, int q_f16, int q_al, float* part, int ks, hipStream_t s) {
     auto* fn = &k_attn_pre<D, NQW>;
     constexpr size_t lds = pre_lds_bytes<D>();
     static_assert(lds <= 160 * 1024, "one workgroup's LDS");
@@ -1548,7 +1539,6 @@ int launch_pre(const AttnArgs& a, int G, int NQ, int q_f16, int q_al, float* par
     });
     if (attr != hipSuccess) return check_hip(attr, "flash_attn_ext: set LDS attribute");
     const int n_qt = (int)cdiv(NQ, 32 * NQW), Hkv = (int)(a.Hq / G);
-    const int ks = pre_splits((int64_t)n_qt * Hkv, cdiv(a.n_kv, 32), 8 / NQW, most);
     hipLaunchKernelGGL(fn, dim3((unsigned)(n_qt * Hkv), (unsigned)ks), dim3(512), lds, s, a, G, NQ, n_qt, q_f16, q_al, ks,
                        ks > 1 ? part : nullptr);
     const int rc = check_hip(hipGetLastError(), "flash_attn_ext (prefill) launch");
@@ -1995,18 +1985,16 @@ int attention(const AttnArgs& a, void* ws, size_t ws_bytes, hipStream_t s) {
 #undef GQ_DEC_U
 #undef GQ_DEC
     } else if (pre_ok(a)) {
-        // query sub-tiles per workgroup: 1 (8 ways over the keys) unless that leaves more than
-        // one workgroup per CU, then 2, then 4
-        const int64_t t32 = cdiv(p.NQ, 32) * a.Hkv;
         const int G = (int)p.G, NQ = (int)p.NQ;
-        const int64_t most = (reinterpret_cast<uintptr_t>(part) & 15) == 0 ? p.n_split : 1;
+        const AttnPrePlan pp =
+            plan_attn_pre(NQ, a.Hkv, a.n_kv, (reinterpret_cast<uintptr_t>(part) & 15) == 0 ? p.n_split : 1);
         if (a.D == 128)
-            return t32 >= 1024 ? launch_pre<128, 4>(b, G, NQ, q_f16, q_al, part, most, s)
-                   : t32 >= 512 ? launch_pre<128, 2>(b, G, NQ, q_f16, q_al, part, most, s)
-                                : launch_pre<128, 1>(b, G, NQ, q_f16, q_al, part, most, s);
-        return t32 >= 1024 ? launch_pre<64, 4>(b, G, NQ, q_f16, q_al, part, most, s)
-               : t32 >= 512 ? launch_pre<64, 2>(b, G, NQ, q_f16, q_al, part, most, s)
-                            : launch_pre<64, 1>(b, G, NQ, q_f16, q_al, part, most, s);
+            return pp.nqw == 4   ? launch_pre<128, 4>(b, G, NQ, q_f16, q_al, part, pp.ks, s)
+                   : pp.nqw == 2 ? launch_pre<128, 2>(b, G, NQ, q_f16, q_al, part, pp.ks, s)
+                                 : launch_pre<128, 1>(b, G, NQ, q_f16, q_al, part, pp.ks, s);
+        return pp.nqw == 4   ? launch_pre<64, 4>(b, G, NQ, q_f16, q_al, part, pp.ks, s)
+               : pp.nqw == 2 ? launch_pre<64, 2>(b, G, NQ, q_f16, q_al, part, pp.ks, s)
+                             : launch_pre<64, 1>(b, G, NQ, q_f16, q_al, part, pp.ks, s);
     } else if (mma_ok(a)) {
         // tiles of 32 query vectors where tiles of 64 leave more than half the CUs idle
         // (Qwen2.5-1.5B shape at 512 tokens, 12 / 2 heads: 96 -> 192 workgroups, 34.1 ->

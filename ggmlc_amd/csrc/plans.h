@@ -96,4 +96,27 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
     return best;
 }
 
+// ---- attention.hip: k_attn_pre (prompt attention)
+
+struct AttnPrePlan {
+    int nqw;  // sub-tiles of 32 queries per workgroup; its 8 waves deal the keys 8 / nqw ways
+    int ks;   // key splits over workgroups
+};
+
+// NQ query vectors per kv head. Sub-tiles: 1 below 512 tiles of 32 query vectors, 2 below 1024,
+// then 4, each longer over the keys but fewer workgroups. 32 / 32 heads, 128 dims, causal, us with
+// 1, 2 and 4: 256 rows (256 tiles) 15.3, 17.2, 21.8; 512 rows 28.6, 22.8, 31.2; 1024 rows 64.8,
+// 49.7, 50.9; 2048 rows 180, 150, 136. Between 257 and 511 tiles 2 would be faster at equal
+// heads (300 rows 25.1, 19.0) and no slower at 12 / 2 (768 rows 25.4, 25.2).
+// Key splits: as many as fill the CUs (one workgroup fills a CU) where each wave would otherwise
+// walk 4 blocks of 32 keys or more, and keeps 2; at most `most`, the splits the caller's
+// workspace holds. The merge is a launch of its own (~4 us).
+inline AttnPrePlan plan_attn_pre(int64_t NQ, int64_t Hkv, int64_t n_kv, int64_t most) {
+    const int64_t t32 = cdiv(NQ, 32) * Hkv;
+    const int nqw = t32 >= 1024 ? 4 : t32 >= 512 ? 2 : 1;
+    const int64_t wgs = cdiv(NQ, 32 * nqw) * Hkv, per_wave = cdiv(n_kv, 32) / (8 / nqw);
+    if (per_wave < 4) return {nqw, 1};
+    return {nqw, (int)std::max<int64_t>(1, std::min<int64_t>({256 / wgs, per_wave / 2, most, 8}))};
+}
+
 }  // namespace gq
