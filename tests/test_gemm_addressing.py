@@ -1,4 +1,5 @@
-"""Host model of the prefill GEMM's addressing (csrc/gemm.hip k_gemm): every global load
+"""Host model of the addressing of the prefill GEMM on fp16 pairs (csrc/gemm.hip k_gemm, weights of an
+odd number of blocks per row; gemm_q8.hip's: test_gemm_q8_model.py): every global load
 offset, LDS address and store index that a launch generates, for the shapes the GPU tests
 and the configs run, checked against the buffer resources, the LDS allocation and the
 output extents on the CPU.
@@ -197,7 +198,7 @@ def workspace_layout(N, K, M):
 
 
 @pytest.mark.parametrize("qt,N,K,M", [(2, 4096, 4096, 512), (2, 96, 11008, 17), (8, 1600, 960, 37), (2, 96, 17408, 17),
-                                     (2, 12288, 4096, 512)])
+                                     (2, 12288, 4096, 512), (2, 12288, 4128, 512), (8, 1600, 992, 37)])
 def test_gemm_workspace_regions_disjoint(qt, N, K, M):
     ws_rs, ws_act, total = workspace_layout(N, K, M)
     assert M * 2 * K * 2 <= ws_rs  # the activation rows end before the row scales
@@ -219,6 +220,10 @@ SHAPES = [
     (2, 32000, 4096, 37), (8, 1600, 960, 512), (8, 5120, 960, 512), (8, 960, 2560, 512),
     (8, 2048, 1536, 16), (8, 17920, 1536, 8), (8, 1536, 8960, 16), (8, 151936, 1536, 7),
     (2, 4096, 4096, 5), (2, 4096, 4096, 129), (8, 256, 512, 70), (2, 96, 64, 3),
+    # odd block counts, which the kernel is reached with (the even ones above address it alike)
+    (2, 64, 1056, 5), (2, 12288, 4128, 512), (2, 4096, 4128, 512), (8, 22016, 4064, 512), (2, 4096, 11040, 512),
+    (8, 1600, 992, 512), (8, 300, 96, 17), (2, 96, 11040, 17), (8, 2048, 2080, 100), (2, 16500, 1056, 130),
+    (8, 16500, 96, 130), (2, 96, 17440, 17), (8, 96, 32, 5),
 ]
 
 
@@ -231,7 +236,7 @@ def test_gemm_addresses_in_bounds(qt, N, K, M):
 
 
 def test_gemm_tail_round_plans():
-    """7B qkv at M = 512: 384 tiles = 256 + 128; the 128 (32 tile columns x 4 token tiles)
+    """12288 rows at M = 512: 384 tiles = 256 + 128; the 128 (32 tile columns x 4 token tiles)
     run with K split 2 ways; gate_up's last round (176 of 256) stays whole"""
     assert launches(12288, 4096, 512) == [(8192, 128, 1, 64), (4096, 128, 2, 32)]
     assert gemm_tail(22016, 4096, 512) is None

@@ -62,3 +62,21 @@ def test_against_block_formula(qt, N, K, M):
     ops.mul_mat(w, x, out=wide[:, :N])
     assert (wide[:, :N].double() - want).abs().max().item() <= tol
     assert (wide[:, N:] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [ops.Q8_0, ops.Q4_0])
+def test_subnormal_scales(qt):
+    """weight and activation scales below 2^-14, where fp16 keeps fewer bits: their products stay exact"""
+    N, K, M = 200, 1088, 40
+    g = torch.Generator(device="cuda")
+    g.manual_seed(qt)
+    b = torch.randint(0, 256, (N, K // 32, ops.BLOCK_BYTES[qt]), generator=g, device="cuda", dtype=torch.uint8)
+    d = (torch.rand((N, K // 32, 1), generator=g, device="cuda") * 5e-5).to(torch.float16)
+    b[..., :2] = d.view(torch.uint8)
+    x = torch.randn((M, K), generator=g, device="cuda") * 1e-3
+    xq = ops.quantize_row_q8_0(x).view(M, K // 32, 34)
+    assert xq[..., :2].contiguous().view(torch.float16).max() < 2.0**-14 and d.max() < 2.0**-14
+    want = _dequant(xq, ops.Q8_0) @ _dequant(b, qt).t()
+    err = ops.mul_mat(ops.QWeight(b.flatten(1).contiguous(), qt, K), x).double() - want
+    assert err.abs().max().item() <= 2.0**-24 * (K // 32) * want.abs().max().item()

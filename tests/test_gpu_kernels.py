@@ -130,8 +130,7 @@ def test_mlp_c2_q4_0(M):
                                    (8960, 1536, 16), (1536, 17920, 12),
                                    # 5..16 rows on int8 MFMA: row tails, K split in 1, 2 and 4 parts
                                    (2048, 100, 9), (4096, 33, 13), (11008, 300, 16), (4096, 16500, 6),
-                                   # a last round of tiles run as its own launch with K split
-                                   # (7B qkv at 512 tokens: 2 ways; Qwen2.5 gate|up: 4 ways)
+                                   # the prefill GEMM on a whole chunk: two and four 32-row tiles a workgroup
                                    (4096, 12288, 512), (1536, 17920, 512)])
 def test_mul_mat_shapes(qtype, K, N, M):
     _check_mm(qtype, K, N, M, seed=K + N + M)
@@ -159,11 +158,11 @@ def _big_rows(M, K, seed):
 @pytest.mark.parametrize("qtype", [O.Q8_0, O.Q4_0])
 @pytest.mark.parametrize("K,N,M", [(4096, 1024, 17), (4096, 1024, 128), (11008, 1024, 512), (11008, 96, 17),
                                    (4096, 300, 3), (4096, 300, 9),
-                                   (17408, 96, 17)])  # K past the one-launch prologue: two-pass row scales
+                                   (17408, 96, 17)])  # K past the one-launch prologue: quantized block by block
 def test_mul_mat_large_activations(qtype, K, N, M):
     """Activation blocks with amax up to 8e6 (where d * q leaves the fp16 range) on every
-    path: the GEMV (M <= 4), int8 MFMA (5..16) and the fp16 MFMA GEMM (row scales, split K at
-    N = 96), within 1e-5 of the oracle and finite."""
+    path: the GEMV (M <= 4), int8 MFMA (5..16) and the prefill GEMM on int8 MFMA (split K at
+    N = 96; the fp16 pairs of odd block counts: test_gemm_odd_blocks.py), within 1e-5 of the oracle and finite."""
     g = torch.Generator(device=DEV)
     g.manual_seed(K + N + M)
     qw = ops.quantize_weights(torch.randn((N, K), generator=g, device=DEV) * 0.02, qtype)
@@ -278,7 +277,7 @@ def test_mul_mat_fused_bit_identical_to_unfused(qtype, K, N, M, rms, glu, add, p
     (O.Q8_0, 1536, 2048, 16, "add_rms"),     # Qwen2.5-1.5B QKV at batch 16 (split K)
     (O.Q8_0, 8960, 1536, 16, "swiglu"),      # Qwen2.5-1.5B down: SWIGLU of gate|up in front
     (O.Q4_0, 11008, 4096, 9, "swiglu"),      # 7B down, 9 rows
-    (O.Q8_0, 960, 960, 5, "add_rms"),        # K = 960 (not a multiple of 64)
+    (O.Q8_0, 960, 960, 5, "add_rms"),        # K = 960 (not a multiple of 256: the prefill GEMM)
     (O.Q4_0, 14336, 64, 6, "rms"),           # K near the prologue's limit
 ])
 def test_mul_mat_fused_gemm_prologue_bit_identical(qtype, K, N, M, mode):
@@ -374,7 +373,7 @@ def test_mul_mat_fused_rope_kv_bit_identical(qtype, K, Hq, Hkv, hd, M, mode, n_d
     (O.Q4_0, 4096, 12288, 37, "gemm"),      # prompt rows: GEMM path, bias in the tile store
     (O.Q8_0, 1536, 17920, 16, "swiglu"),    # batch 16: SWIGLU in the int8 GEMM's epilogue
     (O.Q4_0, 4096, 22016, 6, "swiglu"),     # 6 rows, Q4_0
-    (O.Q8_0, 4096, 12288, 512, "gemm"),     # the last round's rows as a split-K launch: bias offset with them
+    (O.Q8_0, 4096, 12288, 512, "gemm"),     # the prefill GEMM in one part
 ])
 def test_mul_mat_fused_bias_bit_identical(qtype, K, N, M, epi):
     """MUL_MAT with its bias input (executor.cpp:2436-2445: ADD(MUL_MAT(W, x), b)) fused
