@@ -99,8 +99,8 @@ struct GemvFuse {
 int gemv(int type, const uint8_t* W, int64_t N, int64_t K, const ActSrc& act, int64_t M, float* dst, int64_t ldd,
          const GemvFuse& fz, hipStream_t s);
 
-// gemm.hip — dst[m * ldd + n] = rs[m] * sum_k A[m * lda + k] * dequant(W)[n, k] (+ bias[n]),
-// A the fp16 hi + lo rows of the activation prologue and rs its row scales; grids with fewer
+// gemm.hip, for odd block counts — dst[m * ldd + n] = rs[m] * sum_k A[m * lda + k] *
+// dequant(W)[n, k] (+ bias[n]), A the fp16 hi + lo rows of the activation prologue and rs its row scales; grids with fewer
 // tiles than CUs split K over ks workgroups whose partials (part, part_bytes) are summed in
 // order by a second kernel
 struct GemmPlan {
@@ -116,9 +116,9 @@ GemmPlan gemm_plan(int64_t N, int64_t K, int64_t M);
 int gemm(int type, const uint8_t* W, int64_t N, int64_t K, const uint16_t* A, int64_t lda, const float* rs,
          int64_t M, float* dst, int64_t ldd, float* part, hipStream_t s, const float* bias = nullptr);
 
-// gemm_q8.hip — dst[m * ldd + n] (+ bias[n]) for more than GEMM_I8_MAX_M rows on int8 MFMA,
-// from act_prep_q8's layout, for weights whose rows are 4-byte aligned (gemm_q8_ok: K % 64
-// == 0; odd block counts leave rows only 2-byte aligned and take gemm)
+// gemm_q8.hip — dst[m * ldd + n] (+ bias[n]) on int8 MFMA, from act_prep_q8's layout, for weights
+// whose rows are 4-byte aligned (gemm_q8_ok: K % 64 == 0; odd block counts leave rows only 2-byte
+// aligned and take gemm) and every M above GEMV_MAX_M that gemm_i8 does not take
 bool gemm_q8_ok(int64_t K);
 size_t gemm_q8_act_bytes(int64_t K, int64_t M);
 GemmQ8Plan gemm_q8_plan(int type, int64_t N, int64_t K, int64_t M, size_t part_bytes);  // partials within part_bytes
