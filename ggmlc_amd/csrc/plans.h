@@ -54,9 +54,10 @@ inline double fp16_pair_chain(int64_t N, int64_t K, int64_t M, int64_t ncu) {
 // 10.9 in one, 9.9 in two. Segments cost two tiles a workgroup 5 to 7% (how many hardly
 // matters), one tile 1%, or for Q8_0 its third wave per SIMD: 5120 x 960 at 333 tokens (Q4_0)
 // 21.0 us as 2 tiles in two parts, 14.6 as one tile in one part and four segments.
-// A split of at most two tiles a workgroup can sum its stages in segments, the fewest that keep blocks per chain + chains within
-// fp16_pair_chain, so that the error is no larger than in that kernel's order; for Q8_0
-// within 6 more, which its rounded block sums (32 products of 19 bits and more) cost there.
+// Where a split's one chain would pass fp16_pair_chain (for Q8_0 by more than the 6 blocks that its
+// rounded block sums, 32 products of 19 bits and more, cost there), workgroups of at most two tiles
+// sum it in segments, cut where blocks per chain + chains are least (22016 x 4096: 12 + 11 instead
+// of 129): the error is no larger than in that kernel's order, most often far smaller.
 // Partials within part_bytes: split 0 stands in dst, the others in the workspace.
 inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t part_bytes, int64_t ncu) {
     const int64_t nb = K / QK, ns = std::max<int64_t>(1, cdiv(nb, 4)), nt = cdiv(N, 128);
@@ -77,8 +78,15 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
             if (ks != z) continue;  // the same split as a smaller z
             int64_t segs = 1, seg = sps;
             auto chain = [&] { return (double)(std::min<int64_t>(4 * seg, nb) + segs + z - 1); };
-            while (mt <= 2 && seg > 1 && chain() > bound) segs = cdiv(sps, --seg);
-            seg = cdiv(sps, segs);  // as even as they get
+            if (mt <= 2 && chain() > bound) {
+                int64_t least = seg;
+                double c = chain();
+                for (seg = sps; seg >= 1; --seg) {
+                    segs = cdiv(sps, seg);
+                    if (chain() < c) c = chain(), least = seg;
+                }
+                seg = least, segs = cdiv(sps, least);
+            }
             const bool ok = chain() <= bound;
             const int64_t load = cdiv(tiles * ks, ncu), pairs = load / 2;
             const bool three = mt == 1 && load > 1 && (type != GQ_TYPE_Q8_0 || segs == 1);  // registers for 3 waves a SIMD
