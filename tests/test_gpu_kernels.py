@@ -1015,3 +1015,24 @@ def test_calls_without_a_workspace_on_two_streams(call):
     for i in range(2):
         for o in outs[i]:
             assert torch.equal(o, alone[i]), i
+
+
+def test_calls_without_a_workspace_in_a_graph():
+    """the scratch of a captured call is the graph's own: replays between eager calls keep their bits"""
+    g = torch.Generator(device=DEV)
+    g.manual_seed(6)
+    rn = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    q, k, v = rn(12, 128, 128), rn(2, 3072, 128).to(torch.float16), rn(2, 3072, 128).to(torch.float16)
+    w, x = ops.quantize_weights(rn(4096, 4096) * 0.02, O.Q8_0), rn(100, 4096)
+    want = ops.flash_attn_ext(q, k, v, None, 0.1), ops.mul_mat(w, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.flash_attn_ext(q, k, v, None, 0.1), ops.mul_mat(w, x)
+    for _ in range(3):
+        for t in got:
+            t.fill_(float("nan"))
+        graph.replay()
+        ops.flash_attn_ext(q * 2, k, v, None, 0.1), ops.mul_mat(w, x * 2)
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
