@@ -10,7 +10,7 @@ extern "C" void gqbench_gemm_q8_plan(int type, int64_t N, int64_t K, int64_t M, 
 }
 
 extern "C" double gqbench_fp16_pair_chain(int64_t N, int64_t K, int64_t M, int64_t ncu) {
-    return gq::fp16_pair_chain(N, K, M, ncu);
+    return gq::fp16_pair_sums(N, K, M, ncu).chain;
 }
 
 // out: 32-query sub-tiles per workgroup, key splits over workgroups

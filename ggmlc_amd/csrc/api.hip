@@ -88,17 +88,18 @@ int plan_mul_mat(const gq_tensor* a, const gq_tensor* b, const gq_tensor* dst, M
     }
     p.use_gemv = p.M <= GEMV_MAX_M;  // GEMV up to this many activation rows, MFMA GEMM above
     // the GEMV quantizes the activation in LDS; gemm (odd block counts) takes it from the
-    // workspace as the exact fp16 pair hi + lo of d * q / r (rows of 2K halves), then the row scales r (M
-    // floats), followed by the split-K partials when its plan splits K
+    // workspace as the exact fp16 pair hi + lo of d * q / r (rows of 2K halves), then the row
+    // scales r (M floats), followed by the split-K partials when its plan splits K
     p.use_i8 = !p.use_gemv && p.M <= GEMM_I8_MAX_M && K % GEMM_I8_K_ALIGN == 0 && K <= PREP_MAX_K;
     const size_t raw = p.use_gemv ? 0 : (size_t)p.M * K * 4;
     p.ws_rs = (raw + 255) & ~(size_t)255;
     p.ws_act = p.ws_rs + (p.use_gemv ? 0 : (((size_t)p.M * 4 + 255) & ~(size_t)255));
     p.ws = p.ws_act;
-    if (!p.use_gemv && p.M > 0) p.ws += (gemm_plan(N, K, p.M).part_bytes + 255) & ~(size_t)255;
+    p.use_q8 = !p.use_gemv && gemm_q8_ok(K);
+    if (!p.use_gemv && p.M > 0)
+        p.ws += ((p.use_q8 ? gemm_q8_part_bytes(N, K, p.M) : gemm_plan(N, K, p.M).part_bytes) + 255) & ~(size_t)255;
     // gemm_q8 lays its int8 quants and scales (at most 2.2 bytes per element) and then its
     // partials out in the size of that layout, which bounds its K splits
-    p.use_q8 = !p.use_gemv && gemm_q8_ok(K);
     if (p.use_q8) p.ws_act = (gemm_q8_act_bytes(K, p.M) + 255) & ~(size_t)255;
     // the int8 path's activation layout; the GEMM path's size is kept for weights that are
     // not 16-byte aligned (known only at the call), which take the GEMM

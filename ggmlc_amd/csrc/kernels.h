@@ -100,8 +100,8 @@ int gemv(int type, const uint8_t* W, int64_t N, int64_t K, const ActSrc& act, in
          const GemvFuse& fz, hipStream_t s);
 
 // gemm.hip, for odd block counts — dst[m * ldd + n] = rs[m] * sum_k A[m * lda + k] *
-// dequant(W)[n, k] (+ bias[n]), A the fp16 hi + lo rows of the activation prologue and rs its row scales; grids with fewer
-// tiles than CUs split K over ks workgroups whose partials (part, part_bytes) are summed in
+// dequant(W)[n, k] (+ bias[n]), A the fp16 hi + lo rows of the activation prologue and rs its
+// row scales; grids with fewer tiles than CUs split K over ks workgroups whose partials (part, part_bytes) are summed in
 // order by a second kernel
 struct GemmPlan {
     int bm, ks, spk;
@@ -121,6 +121,7 @@ int gemm(int type, const uint8_t* W, int64_t N, int64_t K, const uint16_t* A, in
 // aligned and take gemm) and every M above GEMV_MAX_M that gemm_i8 does not take
 bool gemm_q8_ok(int64_t K);
 size_t gemm_q8_act_bytes(int64_t K, int64_t M);
+size_t gemm_q8_part_bytes(int64_t N, int64_t K, int64_t M);  // the workspace's room for partials
 GemmQ8Plan gemm_q8_plan(int type, int64_t N, int64_t K, int64_t M, size_t part_bytes);  // partials within part_bytes
 int gemm_q8(int type, const uint8_t* W, int64_t N, int64_t K, const uint8_t* A, int64_t M, float* dst, int64_t ldd,
             float* part, size_t part_bytes, hipStream_t s, const float* bias = nullptr);

@@ -17,29 +17,36 @@ struct GemmQ8Plan {
 };
 
 // What bounds the rounding of a product of nb blocks: summed in fp32 chains of n blocks, whose
-// sums are added one after the other, its squared error grows as n + (number of chains). This
-// is that figure for the order in which the fp16-pair kernel (gemm.hip) summed the same
-// product, the yardstick of plan_gemm_q8: K steps of 2 blocks, splits while its tiles of 128
-// rows x 128 or 64 tokens leave CUs idle, and a last partial round of tiles split on its own
-// (there the mean over the rows).
-inline double fp16_pair_chain(int64_t N, int64_t K, int64_t M, int64_t ncu) {
+// sums are added one after the other, its squared error grows as n + (number of chains). `chain`
+// is that figure for the order in which the fp16-pair kernel (gemm.hip) summed such a product
+// when it took all of them, the yardstick of plan_gemm_q8: K steps of 2 blocks, splits while its
+// tiles of 128 rows x 128 or 64 tokens leave CUs idle, and a last partial round of tiles split on
+// its own (there the mean over the rows). `part_bytes` are its partials, the room that the
+// workspace keeps for them. Both stay as they are when that kernel's own plan changes.
+struct Fp16PairSums {
+    double chain;
+    size_t part_bytes;
+};
+inline Fp16PairSums fp16_pair_sums(int64_t N, int64_t K, int64_t M, int64_t ncu) {
     const int64_t nt = cdiv(N, 128), nb = K / QK, nk = cdiv(K, 64);
     const int64_t bm = (M > 64 && nt >= 16) || nt * cdiv(M, 128) >= ncu ? 128 : 64;
     const int64_t mtiles = cdiv(M, bm), tiles = nt * mtiles;
-    auto chain = [&](int64_t ks) {
-        const int64_t spk = cdiv(nk, std::max<int64_t>(1, ks));
-        return (double)(std::min<int64_t>(2 * spk, nb) + cdiv(nk, spk));
+    auto sums = [&](int64_t want, int64_t rows) {  // `rows` weight rows in about `want` splits
+        const int64_t spk = cdiv(nk, std::max<int64_t>(1, want)), ks = cdiv(nk, spk);
+        return Fp16PairSums{(double)(std::min<int64_t>(2 * spk, nb) + ks),
+                            ks > 1 ? (size_t)ks * M * rows * sizeof(float) : 0};
     };
-    if (tiles < ncu) return chain(std::min<int64_t>({cdiv((bm == 128 ? 1 : 2) * ncu, tiles), nk / 4, 16}));
+    if (tiles < ncu) return sums(std::min<int64_t>({cdiv((bm == 128 ? 1 : 2) * ncu, tiles), nk / 4, 16}), N);
     if (bm == 128 && tiles > ncu && ncu % mtiles == 0) {
         const int64_t head = tiles / ncu * (ncu / mtiles), tail = (nt - head) * mtiles;
         const int64_t kt = tail > 0 && 2 * tail <= ncu ? std::min<int64_t>({ncu / tail, nk / 4, 4}) : 1;
         if (kt >= 2) {
             const double f = (double)(head * 128) / (double)N;
-            return f * chain(1) + (1.0 - f) * chain(kt);
+            const Fp16PairSums t = sums(kt, N - head * 128);
+            return {f * sums(1, N).chain + (1.0 - f) * t.chain, t.part_bytes};
         }
     }
-    return chain(1);
+    return sums(1, N);
 }
 
 // Tiles of 32 mt tokens, ks K splits: the pair with the shortest expected launch. Measured per
@@ -54,7 +61,7 @@ inline double fp16_pair_chain(int64_t N, int64_t K, int64_t M, int64_t ncu) {
 // 10.9 in one, 9.9 in two. Segments cost two tiles a workgroup 5 to 7% (how many hardly
 // matters), one tile 1%, or for Q8_0 its third wave per SIMD: 5120 x 960 at 333 tokens (Q4_0)
 // 21.0 us as 2 tiles in two parts, 14.6 as one tile in one part and four segments.
-// Where a split's one chain would pass fp16_pair_chain (for Q8_0 by more than the 6 blocks that its
+// Where a split's one chain would pass fp16_pair_sums (for Q8_0 by more than the 6 blocks that its
 // rounded block sums, 32 products of 19 bits and more, cost there), workgroups of at most two tiles
 // sum it in segments, cut where blocks per chain + chains are least (22016 x 4096: 12 + 11 instead
 // of 129): the error is no larger than in that kernel's order, most often far smaller.
@@ -66,7 +73,7 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
     if (slab > 0) most += (int64_t)((double)part_bytes / slab);
     most = std::min<int64_t>({most, std::max<int64_t>(1, ns / 3), 16});  // at least 3 stages each
     most = cdiv(ns, cdiv(ns, most));  // the splits that many leave non-empty
-    const double bound = fp16_pair_chain(N, K, M, ncu) + (type == GQ_TYPE_Q8_0 ? 6.0 : 0.0);
+    const double bound = fp16_pair_sums(N, K, M, ncu).chain + (type == GQ_TYPE_Q8_0 ? 6.0 : 0.0);
     GemmQ8Plan best{1, 1, (int)ns, (int)ns};
     double best_us = 1e300;
     bool best_ok = false;
@@ -81,9 +88,9 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
             if (mt <= 2 && chain() > bound) {
                 int64_t least = seg;
                 double c = chain();
-                for (seg = sps; seg >= 1; --seg) {
+                for (seg = 1; seg < sps && seg * seg <= 2 * sps; ++seg) {  // (least near sqrt(sps / 4))
                     segs = cdiv(sps, seg);
-                    if (chain() < c) c = chain(), least = seg;
+                    if (chain() <= c) c = chain(), least = seg;
                 }
                 seg = least, segs = cdiv(sps, least);
             }
