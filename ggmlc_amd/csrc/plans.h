@@ -61,10 +61,12 @@ inline Fp16PairSums fp16_pair_sums(int64_t N, int64_t K, int64_t M, int64_t ncu)
 // 10.9 in one, 9.9 in two. Segments cost two tiles a workgroup 5 to 7% (how many hardly
 // matters), one tile 1%, or for Q8_0 its third wave per SIMD: 5120 x 960 at 333 tokens (Q4_0)
 // 21.0 us as 2 tiles in two parts, 14.6 as one tile in one part and four segments.
-// Where a split's one chain would pass fp16_pair_sums (for Q8_0 by more than the 6 blocks that its
-// rounded block sums, 32 products of 19 bits and more, cost there), workgroups of at most two tiles
-// sum it in segments, cut where blocks per chain + chains are least (22016 x 4096: 12 + 11 instead
-// of 129): the error is no larger than in that kernel's order, most often far smaller.
+// Where a split's one chain would pass fp16_pair_sums (in Q8_0, whose block sums, 32 products of 19
+// bits and more, round there, up to 6 blocks more while that is no more than 20), workgroups of at
+// most two tiles sum it in segments, cut where blocks per chain + chains are least (22016 x 4096: 12 + 11 instead
+// of 129): the error is no larger than in that kernel's order, most often far smaller. The two
+// kinds are timed less alike than this model says, so segments have to save a sixth where whole
+// splits keep the bound too.
 // Partials within part_bytes: split 0 stands in dst, the others in the workspace.
 inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t part_bytes, int64_t ncu) {
     const int64_t nb = K / QK, ns = std::max<int64_t>(1, cdiv(nb, 4)), nt = cdiv(N, 128);
@@ -73,10 +75,10 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
     if (slab > 0) most += (int64_t)((double)part_bytes / slab);
     most = std::min<int64_t>({most, std::max<int64_t>(1, ns / 3), 16});  // at least 3 stages each
     most = cdiv(ns, cdiv(ns, most));  // the splits that many leave non-empty
-    const double bound = fp16_pair_sums(N, K, M, ncu).chain + (type == GQ_TYPE_Q8_0 ? 6.0 : 0.0);
-    GemmQ8Plan best{1, 1, (int)ns, (int)ns};
-    double best_us = 1e300;
-    bool best_ok = false;
+    double bound = fp16_pair_sums(N, K, M, ncu).chain;
+    if (type == GQ_TYPE_Q8_0) bound = std::max(bound, std::min(bound + 6.0, 20.0));
+    GemmQ8Plan whole{1, 1, (int)ns, (int)ns}, cut = whole;
+    double whole_us = 1e300, cut_us = 1e300;
     for (int mt = (int)std::max<int64_t>(1, std::min<int64_t>(4, cdiv(M, 32))); mt >= 1; --mt) {
         const int64_t tiles = nt * cdiv(M, 32 * mt);
         const double one = 0.56 + 0.245 * mt, two = 0.53 + 0.485 * mt;
@@ -94,21 +96,18 @@ inline GemmQ8Plan plan_gemm_q8(int type, int64_t N, int64_t K, int64_t M, size_t
                 }
                 seg = least, segs = cdiv(sps, least);
             }
-            const bool ok = chain() <= bound;
+            if (chain() > bound) continue;
             const int64_t load = cdiv(tiles * ks, ncu), pairs = load / 2;
             const bool three = mt == 1 && load > 1 && (type != GQ_TYPE_Q8_0 || segs == 1);  // registers for 3 waves a SIMD
             double us = (double)sps * (three ? 0.5 * (double)load : pairs * two + (load & 1) * one);
             if (mt > 1) us += 3.0 * (double)((load - 1) / 2);  // a further round's first loads and last stores
             if (mt == 2 && segs > 1) us *= 1.06;
             if (ks > 1) us += 2.5 + slab * 2 * (double)ks / 6e6;
-            if ((ok && !best_ok) || (ok == best_ok && us < best_us)) {
-                best_us = us;
-                best_ok = ok;
-                best = GemmQ8Plan{mt, (int)ks, (int)sps, (int)seg};
-            }
+            if (segs == 1 && us < whole_us) whole_us = us, whole = GemmQ8Plan{mt, (int)ks, (int)sps, (int)seg};
+            if (segs > 1 && us < cut_us) cut_us = us, cut = GemmQ8Plan{mt, (int)ks, (int)sps, (int)seg};
         }
     }
-    return best;
+    return whole_us <= 1.2 * cut_us ? whole : cut;
 }
 
 // ---- attention.hip: k_attn_pre (prompt attention)

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from ggmlc_amd import ops
-from test_gemm_q8_model import bench_lib, plan
+from test_gemm_q8_model import bench_lib, chain_bound, plan
 
 SHAPES = [
     (130, 512, 17), (131, 4096, 40),  # one 32-row tile; splits, rows not 16-byte aligned
@@ -55,7 +55,7 @@ def test_against_block_formula(qt, N, K, M):
     # c roundings of partial sums that grow like a random walk: each of variance ulp^2 / 12, ulp^2
     # on average 0.57 (2^-23)^2 of the square, c / 2 of the final sum's square in all; 1.1 for c's
     # own spread over the shapes
-    c = bench_lib().gqbench_fp16_pair_chain(N, K, M, 256) + (6 if qt == ops.Q8_0 else 0)
+    c = chain_bound(qt, bench_lib().gqbench_fp16_pair_chain(N, K, M, 256))
     assert (err.norm() / want.norm()).item() <= 1.1 * 2.0**-23 * (c / 2 * 0.57 / 12) ** 0.5
     # rows of a wider buffer: split 0's slab keeps to its columns
     wide = torch.full((M, N + 5), 7.0, device="cuda")
